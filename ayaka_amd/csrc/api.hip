@@ -219,9 +219,19 @@ int wave_split_for(const ayk::AttnParams& p, bool split, int32_t flags) {
 // reduce kernel (no wave split, no single launch, no q.k choice).
 int launch_f32(const char* op, const ayk::AttnParams& p, int head_dim, int gc, bool split, int32_t flags,
                void* stream) {
+  if (!split && flags == AYK_FLAG_ROW_TILES && p.positions) {
+    if ((int64_t)p.n_rows * p.num_heads > INT32_MAX)
+      return fail(AYK_ERR_UNSUPPORTED, "%s: %d rows of %d heads exceed one launch", op, p.n_rows, p.num_heads);
+    if (ayk::walking()) {
+      ayk::walk_rows_f32(p, head_dim, compute_units());
+      return ok();
+    }
+    return launched(ayk::launch_rows_f32(p, head_dim, compute_units(), static_cast<hipStream_t>(stream)), op);
+  }
   if (flags & ~(AYK_FLAG_PARTIALS_ONLY | AYK_FLAG_SEPARATE_REDUCE | AYK_FLAG_WAVES_1))
     return fail(AYK_ERR_UNSUPPORTED, "%s: flags 0x%x: fp32 runs one kernel shape (partials only, a separate "
-                "reduce and one wave per head are the flags it takes)", op, flags);
+                "reduce and one wave per head are the flags it takes; v1 also row tiles alone, over rows with "
+                "positions)", op, flags);
   ayk::AttnParams q = p;
   q.wave_split = 1;
   q.arrivals = nullptr;

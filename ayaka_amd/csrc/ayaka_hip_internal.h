@@ -73,6 +73,8 @@ hipError_t launch_window_mfma(const AttnParams& p, int head_dim, bool bf16, bool
 // fp32 models: the VALU decode kernel (v1, or v2 partitions) and its partition merge.
 hipError_t launch_attention_f32(const AttnParams& p, int head_dim, int heads_per_chunk, bool split,
                                 hipStream_t stream);
+// fp32 models, multi-row steps: rows (with positions) in tiles that share their request's reads.
+hipError_t launch_rows_f32(const AttnParams& p, int head_dim, int compute_units, hipStream_t stream);
 hipError_t launch_partition_reduce_f32(const AttnParams& p, int head_dim, int compute_units, hipStream_t stream);
 // The v2 log-sum-exp merge of the partitions of every (row, head); `compute_units` of the
 // device sets how many partition slots each pair gets.
@@ -85,6 +87,7 @@ hipError_t launch_row_reduce(const AttnParams& p, int head_dim, bool bf16, hipSt
 bool walking();
 void walk_decode(const AttnParams& p, int head_dim, bool mfma, bool kv8, bool split, bool window);
 void walk_f32(const AttnParams& p, int head_dim, bool split);
+void walk_rows_f32(const AttnParams& p, int head_dim, int compute_units);
 void walk_prefill(const AttnParams& p, const int32_t* tiles, int n_tiles, int head_dim, bool kv8,
                   int waves_per_group);
 

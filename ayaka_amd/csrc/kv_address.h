@@ -116,6 +116,19 @@ constexpr int f32_floats_per_lane(int gc) { return AYK_F32_WIDE_GC < gc ? 8 : 4;
 constexpr int f32_lanes_per_position(int d, int gc) { return d / f32_floats_per_lane(gc); }
 constexpr int f32_loads_per_chunk(int gc) { return f32_floats_per_lane(gc) == 8 ? 2 : 4; }
 
+// Multi-row kernel over fp32 caches: 16-position steps, W waves of a workgroup taking every W-th
+// (4 where two waves per SIMD would not hold the registers), and 16-pair groups per tile: two
+// where the grid still covers the compute units twice over (each key and value load then feeds
+// twice the products), else one.
+constexpr int rows_f32_step() { return 16; }
+constexpr int rows_f32_waves(int d, int groups) { return d == 256 || (d == 128 && groups == 2) ? 4 : 8; }
+AYK_HD int64_t rows_f32_tiles(const AttnParams& p, int groups) {
+  return ((int64_t)p.n_rows * p.group + 16 * groups - 1) / (16 * groups);
+}
+AYK_HD int rows_f32_groups(const AttnParams& p, int d, int compute_units) {
+  return d != 256 && rows_f32_tiles(p, 2) * (p.num_heads / p.group) >= 2 * (int64_t)compute_units ? 2 : 1;
+}
+
 // Multi-row kernel: 64-position chunks, or 32 at head_dim 256 with 1 or 2 waves per pair group
 // (a 64-position stage there took 133 KB of LDS and left one wave per SIMD).
 constexpr int prefill_chunk_positions(int d, int waves_per_group) { return d == 256 && waves_per_group <= 2 ? 32 : 64; }

@@ -225,6 +225,49 @@ void walk_f32_d(const AttnParams& p, bool split) {
     }
 }
 
+// The multi-row kernel over fp32 caches: a tile's rows request by request, each wave's steps.
+template <int D>
+void walk_rows_f32_d(const AttnParams& p, int groups) {
+  constexpr int CH = rows_f32_step();
+  const int waves = rows_f32_waves(D, groups);
+  const uint32_t token_stride = (uint32_t)p.token_stride;
+  std::vector<uint32_t> buffer;
+  const int pairs = 16 * groups, n_pairs = p.n_rows * p.group;
+  for (int64_t tile = 0; tile < rows_f32_tiles(p, groups); ++tile) {
+    std::vector<std::pair<int, int>> spans;  // (request, the longest context among its rows of the tile)
+    for (int pair = (int)tile * pairs; pair < std::min<int64_t>(n_pairs, (tile + 1) * pairs); ++pair) {
+      int req, len;
+      row_of(p, pair / p.group, req, len);
+      auto at = std::find_if(spans.begin(), spans.end(), [&](const auto& s) { return s.first == req; });
+      if (at == spans.end()) spans.push_back({req, len});
+      else at->second = std::max(at->second, len);
+    }
+    for (const auto& [req, t_end] : spans)
+      for (int kvh = 0; kvh < p.num_heads / p.group; ++kvh) {
+        const int seg_len = segment_positions(p, CH);
+        for (int s0 = 0; s0 < t_end; s0 += seg_len) {
+          const int s1 = imin(t_end, s0 + seg_len);
+          const int b0 = stage(p, (int64_t)req * p.table_stride, s0, s1, buffer);
+          const int nch = (s1 - s0 + CH - 1) / CH;
+          for (int wave = 0; wave < waves && wave < nch; ++wave)
+            for (int ci = wave; ci <= last_chunk_of_slice(nch, wave, waves); ci += waves)
+              for (int lane = 0; lane < 64; ++lane) {
+                const int mt = lane % 16, mq = lane / 16;
+                const uint32_t k = kv_offset(p, buffer.data() + kTableCap, b0,
+                                             chunk_position(s0, s1, ci, CH, 0, CH, mt), token_stride);
+                for (int u = 0; u < D / 16; ++u)
+                  record(4 * ((int64_t)kvh * p.head_stride + 4 * mq + (int64_t)k + 16 * u), 16);
+                uint32_t off[4];
+                prefill_offsets<4>(p, buffer.data() + kTableCap, b0, s0 + ci * CH + 4 * mq, s1, 0, token_stride, off);
+                for (int i = 0; i < 4; ++i)
+                  for (int c = 0; c < D / 64; ++c)
+                    record(4 * ((int64_t)kvh * p.head_stride + 4 * mt + (int64_t)off[i] + 64 * c), 16);
+              }
+        }
+      }
+  }
+}
+
 template <int D, bool KV8, int PS, int N, int THREADS>
 void walk_prefill_typed(const AttnParams& p, const int32_t* tiles, int n_tiles) {
   constexpr int CH = prefill_chunk_positions(D, PS);
@@ -313,6 +356,15 @@ void walk_f32(const AttnParams& p, int head_dim, bool split) {
   // the kernel's lane geometry depends only on whether its heads per wave take the wide rows
   if (f32_floats_per_lane(p.group / p.head_chunks) == 8) walk_f32_gc<8>(p, head_dim, split);
   else walk_f32_gc<1>(p, head_dim, split);
+}
+
+void walk_rows_f32(const AttnParams& p, int head_dim, int compute_units) {
+  const int groups = rows_f32_groups(p, head_dim, compute_units);
+  switch (head_dim) {
+    case 64: walk_rows_f32_d<64>(p, groups); break;
+    case 128: walk_rows_f32_d<128>(p, groups); break;
+    default: walk_rows_f32_d<256>(p, groups); break;
+  }
 }
 
 void walk_prefill(const AttnParams& p, const int32_t* tiles, int n_tiles, int head_dim, bool kv8,

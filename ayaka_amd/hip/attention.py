@@ -134,6 +134,8 @@ PARTIALS_ONLY = 4
 _MERGE_FLAGS = {None: 0, "reduce-kernel": 8, "in-kernel": 16}
 #: AYK_FLAG_WAVES_*: waves sharing each (row, key/value head)'s context (v1) or partition (v2)
 _WAVE_FLAGS = {None: 0, 1: 32, 2: 64, 4: 128, 8: 256}
+#: AYK_FLAG_ROW_TILES: v1 over fp32 rows in tiles that share their request's reads
+ROW_TILES = 512
 
 
 @dataclass(frozen=True, slots=True)
@@ -241,6 +243,17 @@ class HipAttentionPlan:
                 if best is None or t < best[0] * (1 - PREFILL_SMALLER_TILE_MARGIN):
                     best = (t, pairs, size)
             found = (best[1], best[2])
+            self.splits[key] = found
+        return found
+
+    def row_tiles(self, num_kv_heads: int, group: int, head_dim: int) -> bool:
+        """Whether an fp32 multi-row step runs in tiles of rows (chosen once for every layer)."""
+        key = ("row-tiles", num_kv_heads, group, head_dim)
+        found = self.splits.get(key)
+        if found is None:
+            live = [count for count, length in zip(self.rows, self.kv_lengths) if count and length]
+            found = bool(live) and row_tiles_faster(live, self.max_length, sum(self.row_lengths), num_kv_heads, group,
+                                                    head_dim)
             self.splits[key] = found
         return found
 
@@ -792,6 +805,39 @@ def prefill_model_us(group_lengths: list[int], row_lengths: tuple[int, ...] | li
     return t
 
 
+#: An fp32 step in tiles of rows (``paged_rows_f32_kernel``), modelled: a workgroup's fixed time, the
+#: time of one 16-position step of each of its waves by head width and 16-pair groups per tile, and
+#: the rate (flops per us) of a launch that fills the GPU. Row by row: a fixed time and the rate
+#: (bytes per us) at which every row streams its own context. Fitted to 60 steps (3 and 8 key/value
+#: heads, GQA 2 to 8, head widths 64 to 256, 2 to 2000 rows over 64 to 8192 positions), measured both
+#: ways: the faster side was taken on all but three, whose two sides are within 20%.
+ROW_TILES_FIXED_US = 6.0
+ROW_TILES_STEP_US = {(64, 1): 1.5, (64, 2): 3.0, (128, 1): 2.9, (128, 2): 3.6, (256, 1): 2.9}
+ROW_TILES_FLOPS_PER_US = 8.0e7
+ROWS_FIXED_US = 10.0
+ROWS_BYTES_PER_US = 8.0e6
+#: How much faster the tiles must model (their work depends more on how rows fall into tiles).
+ROW_TILES_MARGIN = 1.15
+
+
+def row_tiles_faster(rows: list[int], longest: int, total: int, num_kv_heads: int, group: int, head_dim: int) -> bool:
+    """Whether an fp32 multi-row step models faster in tiles of rows than row by row: ``rows`` the
+    rows of its requests with context, ``longest`` the longest context and ``total`` the sum of
+    its rows' contexts. A tile holds 16 or 32 consecutive (row, query head) pairs and walks its
+    requests one after the other, so short requests cost it their contexts in turn."""
+    pairs = sum(rows) * group
+    groups = 2 if head_dim != 256 and -(-pairs // 32) * num_kv_heads >= 2 * COMPUTE_UNITS else 1
+    waves = 4 if head_dim == 256 or (head_dim == 128 and groups == 2) else 8
+    tile, least = 16 * groups, min(rows) * group
+    aligned = all(count * group % tile == 0 for count in rows)
+    requests = min(len(rows), -(-tile // least) if aligned or least < tile and tile % least == 0
+                   else 1 + -(-(tile - 1) // least))
+    chain = requests * -(-longest // (16 * waves)) * ROW_TILES_STEP_US[(head_dim, groups)]
+    tiles = ROW_TILES_FIXED_US + max(chain, 4 * num_kv_heads * group * head_dim * total / ROW_TILES_FLOPS_PER_US)
+    by_row = ROWS_FIXED_US + total * num_kv_heads * 2 * head_dim * 4 / ROWS_BYTES_PER_US
+    return tiles * ROW_TILES_MARGIN < by_row
+
+
 def choose_prefill_partition(group_lengths: list[int], row_lengths: tuple[int, ...] | list[int],
                              num_kv_heads: int, num_heads: int, head_dim: int, waves_per_group: int = 1,
                              context_bytes: int = 0) -> int:
@@ -1024,8 +1070,13 @@ def attend_with(
 
     lib = _lib.lib()
     stream = stream_handle(device)
+    row_tiles = False
     if q.dtype == torch.float32:
-        # fp32 models run on the decode kernel for fp32, each row of a multi-row step on its own
+        # fp32 models run on the decode kernel for fp32, each row of a multi-row step on its own,
+        # or in tiles of rows that share their request's reads when the launch is left to the library
+        row_tiles = (partitions is None and prefill is None and not decode and isinstance(step, HipAttentionPlan)
+                     and not partials_only and merge is None and waves is None
+                     and step.row_tiles(kv_heads, heads // kv_heads, buffers.head_dim))
         if prefill or window or (qk is not None) or (waves not in (None, 1)) or merge == "in-kernel":
             raise BackendError(f"{op}: fp32 runs one launch shape: the per-row decode kernel, one wave per "
                                "head, partitions merged by the reduce kernel", context={"op": op})
@@ -1106,6 +1157,9 @@ def attend_with(
         float(scale),
         *codec_scales(buffers.codec),
     )
+    if row_tiles:
+        _call(op, lib.ayk_paged_attention_v1, (*common, ROW_TILES), stream, device, False, _record)
+        return
     staged = None
     if partitions is None:
         kv_bytes = buffers.k.element_size()

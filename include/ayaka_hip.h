@@ -44,7 +44,8 @@ enum {
  * byte per element, decoded exactly to the compute dtype when read; AYK_DTYPE_FP32
  * for fp32 models (q, out and caches all fp32; decode entry points only, on the VALU:
  * ayk_paged_attention_v1 / _v2 / _v2_static, whose rows may carry positions, so a
- * multi-row step runs row by row; the window and multi-row entry points refuse it). */
+ * multi-row step runs row by row, or in tiles of rows with AYK_FLAG_ROW_TILES; the window and
+ * multi-row entry points refuse it). */
 enum { AYK_DTYPE_FP16 = 0, AYK_DTYPE_BF16 = 1, AYK_DTYPE_FP8_E4M3 = 2, AYK_DTYPE_FP32 = 3 };
 
 /* flags of the attention calls: 0 lets the library pick the q.k path. */
@@ -62,7 +63,10 @@ enum {
   AYK_FLAG_WAVES_1 = 32,
   AYK_FLAG_WAVES_2 = 64,
   AYK_FLAG_WAVES_4 = 128,
-  AYK_FLAG_WAVES_8 = 256
+  AYK_FLAG_WAVES_8 = 256,
+  AYK_FLAG_ROW_TILES = 512 /* v1 over fp32 rows that carry positions: consecutive rows of a request share its
+                              context's reads, q.k and P.V on the matrix cores in fp32 (for steps of many rows
+                              per request; rows of one request need not be adjacent, but only those share) */
 };
 enum { AYK_LAYOUT_NHD = 0, AYK_LAYOUT_HND = 1 };
 

@@ -1,0 +1,117 @@
+"""fp32 multi-row steps in tiles of rows (``AYK_FLAG_ROW_TILES``): prompts and prefill chunks.
+
+The kernel is compared with the float64 oracle at the sizes where it can go wrong: groups that do and do
+not divide a tile, tiles that span requests, contexts around its 16-position steps and its wave split,
+block sizes that take one table lookup per step and those that do not, and values that are not finite
+where only some rows of a tile see them. The bound is the reference contract's for fp32,
+``4 * eps * max|y| + 1e-6``.
+"""
+
+from __future__ import annotations
+
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from ayaka_amd.enums import ForwardMode, KVLayoutKind
+from ayaka_amd.hip import _lib
+from ayaka_amd.hip import attention as hip_attention
+from ayaka_amd.kvcache import RAW_CODEC, KVBuffers
+from tests import test_kv_reach as reach
+from tests._support import build_scenario
+
+EPS32 = 2.0**-23
+
+# (rows, context) of each request
+STEPS = [
+    [(16, 16)],
+    [(8, 8), (9, 40), (31, 31), (12, 300)],
+    [(150, 150), (8, 1000), (10, 0), (33, 129)],
+    [(300, 700)],
+]
+
+
+@pytest.mark.parametrize("head_dim", [64, 128, 256])
+def test_row_tiles_read_inside_the_cache(head_dim: int) -> None:
+    rng = np.random.default_rng(700 + head_dim)
+    for case in range(10):
+        bs = reach.BLOCK_SIZES[case % len(reach.BLOCK_SIZES)]
+        kv_heads, group = [(2, 4), (3, 3), (1, 20), (4, 1)][case % 4]
+        lengths = [int(n) for n in rng.integers(1, 300, size=int(rng.integers(1, 4)))]
+        step = reach.Step(rng, lengths, bs, kv_heads, head_dim, False, case % 2, fp32=True)
+        rows = [max(1, n // 3) for n in lengths]
+        req, pos = reach._rows(step, rows)
+        args = reach._common(step, kv_heads * group, len(req), req, pos)
+        got = reach._walk(step, lambda lib: lib.ayk_paged_attention_v1(*args, hip_attention.ROW_TILES, None))
+        reach._check(step, got, f"row tiles case {case} bs {bs}")
+
+
+def test_row_tiles_are_refused_elsewhere() -> None:
+    lib = _lib.lib()
+
+    def v1(dtype: int, flags: int, rows: object) -> int:
+        return lib.ayk_paged_attention_v1(1, 1, 1, 1, 1, 4, 1, rows, rows, 1, 8, 2, 128, 10, 16, 4, 0, dtype, dtype,
+                                          ctypes.c_float(1.0), 1.0, 1.0, flags, None)
+
+    assert v1(1, hip_attention.ROW_TILES, 1) == 1 and b"unknown flags" in lib.ayk_last_error()
+    assert v1(3, hip_attention.ROW_TILES, None) == 2 and b"rows with positions" in lib.ayk_last_error()
+    assert v1(3, hip_attention.ROW_TILES | 32, 1) == 2
+
+
+def _f32(a: np.ndarray) -> torch.Tensor:
+    return torch.from_numpy(np.ascontiguousarray(a, dtype=np.float32)).to("cuda:0")
+
+
+def _planned(steps, heads: int, kv_heads: int, head_dim: int, block_size: int, layout: str, seed: int):
+    s = build_scenario(steps, heads=heads, kv_heads=kv_heads, head_dim=head_dim, block_size=block_size,
+                       layout=layout, mode="mixed", seed=seed)
+    meta = hip_attention.plan(ForwardMode.MIXED, torch.tensor(s.rows, dtype=torch.int32, device="cuda:0"),
+                              torch.tensor(s.lengths, dtype=torch.int32, device="cuda:0"),
+                              torch.from_numpy(s.table.astype(np.int32)).cuda(), block_size)
+    buffers = KVBuffers(_f32(s.k), _f32(s.v), KVLayoutKind.NHD if layout == "nhd" else KVLayoutKind.HND, RAW_CODEC)
+    return s, meta, buffers, _f32(s.q)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,kv_heads,head_dim", [(9, 3, 64), (32, 8, 64), (8, 2, 128), (5, 5, 128), (20, 1, 128),
+                                                     (16, 8, 256), (6, 2, 256)])
+@pytest.mark.parametrize("block_size,layout", [(16, "nhd"), (24, "hnd"), (5, "nhd"), (1, "hnd")])
+def test_row_tiles_match_the_oracle(heads: int, kv_heads: int, head_dim: int, block_size: int, layout: str) -> None:
+    for n, steps in enumerate(STEPS):
+        s, meta, buffers, q = _planned(steps, heads, kv_heads, head_dim, block_size, layout, 710 + n)
+        assert meta.plan.row_tiles(kv_heads, heads // kv_heads, head_dim), steps
+        expected = s.expected(np.float64)
+        out = torch.full_like(q, 7.0)
+        for _ in range(2):  # recorded, then replayed
+            hip_attention.attend(q, buffers, meta, out, scale=s.scale)
+        torch.cuda.synchronize()
+        got = out.double().cpu().numpy()
+        bound = 4 * EPS32 * float(np.abs(expected).max()) + 1e-6
+        assert np.isfinite(got).all(), steps
+        assert float(np.abs(got - expected).max()) <= bound, steps
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("head_dim", [64, 256])
+def test_values_that_are_not_finite_reach_only_the_rows_that_see_them(head_dim: int) -> None:
+    s, meta, buffers, q = _planned([(40, 70)], 8, 2, head_dim, 16, "nhd", 720)
+    clean, out = torch.empty_like(q), torch.empty_like(q)
+    hip_attention.attend(q, buffers, meta, clean, scale=s.scale)
+    at = 53  # positions 30 to 69 are the rows; rows before position 53 do not see it
+    block, offset = int(s.table[0][at // 16]), at % 16
+    buffers.v[block, offset, 0, 3] = float("inf")
+    buffers.v[block, offset, 1, 5] = float("nan")
+    hip_attention.attend(q, buffers, meta, out, scale=s.scale)
+    torch.cuda.synchronize()
+    before = at - 30
+    # a step with such a value sums its positions one by one, in another order than the clean one:
+    # the contract's bound on each side of the exact result
+    bound = 2 * (4 * EPS32 * float(clean.abs().max()) + 1e-6)
+    assert float((out[:before] - clean[:before]).abs().nan_to_num(float("inf")).max()) <= bound
+    assert torch.isinf(out[before:, :4, 3]).all() and torch.isnan(out[before:, 4:, 5]).all()
+    kept = torch.ones(head_dim, dtype=torch.bool, device="cuda:0")
+    kept[3] = False
+    others = (out[before:, :4] - clean[before:, :4])[:, :, kept]
+    assert float(others.abs().nan_to_num(float("inf")).max()) <= bound
