@@ -233,7 +233,8 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void paged_attention_mfma_kernel
     // accesses running in program order), the SUB independent score tiles then take one
     // max, one rescale decision and one pass of exponentials, and the values follow tile
     // by tile for P.V.
-    auto consume = [&](int ci, const Raw(&kc)[NL], const Raw(&vc)[NL]) {
+    // keys_used() runs once the keys are in LDS or spent, values_used() once the values are.
+    auto consume = [&](int ci, const Raw(&kc)[NL], const Raw(&vc)[NL], auto&& keys_used, auto&& values_used) {
       const int tc = s0 + ci * CH;
       const bool tail = tc + CH > s1;
       f32x4 acc[SUB];
@@ -246,6 +247,7 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void paged_attention_mfma_kernel
 #pragma unroll
         for (int s = 0; s < KS; ++s) acc[sub] = mfma_qk<BF16>(s_k[wave][key_slot(mt, s * 4 + mq)], qb[s], acc[sub]);
       }
+      keys_used();
       float mx = -INFINITY;
 #pragma unroll
       for (int sub = 0; sub < SUB; ++sub)
@@ -289,6 +291,7 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void paged_attention_mfma_kernel
         for (int j = 0; j < NL1; ++j)
           *reinterpret_cast<u32x4*>(&s_v[wave][(j * TPL + r) * VP + c * 8]) = kv_pairs<KV8, PB>(vc[sub * NL1 + j]);
         wave_lds_sync();
+        if (sub == SUB - 1) values_used();
 #pragma unroll
         for (int t = 0; t < DT; ++t) {
           const u32x2 va = lds_read_transposed(&s_v[wave][(4 * mq + (mt >> 2)) * VP + t * 16 + 4 * (mt & 3)]);
@@ -298,33 +301,60 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void paged_attention_mfma_kernel
       }
     };
 
-    // Keys of the next chunk are in flight while the current one is folded in. The
-    // prefetch is unconditional -- at the last chunk it re-reads that chunk, which
-    // has just arrived -- so the compiler's waits for the values before each use
-    // leave the next chunk's keys outstanding (a conditional load would make them
-    // wait for everything).
-    uint32_t offA[NL], offB[NL];
-    Raw kA[NL], kB[NL], vc[NL];
+    uint32_t offA[NL];
+    Raw kA[NL], vc[NL];
     int ci = slice;
     offsets(ci, offA);
 #pragma unroll
     for (int j = 0; j < NL; ++j) kA[j] = load_kv_raw<KV8>(kbase, offA[j]);
-    while (ci <= last) {
+    if constexpr (D == 256) {
+      // One buffer each for keys and values, refilled with the next chunk's as soon as this
+      // chunk's are in LDS (at the last chunk: that chunk again). With the two key buffers
+      // below this width took 54-113 registers more than two waves per SIMD have, and the
+      // spills bounded every chunk: 16/8 heads, us, before -> now: 32 rows of 4000 positions
+      // 241 -> 165 (6.4 TB/s), over fp8 caches 120 -> 87; 1 row of 500 28 -> 18; 4-row windows
+      // over 64 contexts of 1500 202 -> 124.
 #pragma unroll
       for (int j = 0; j < NL; ++j) vc[j] = load_kv_raw<KV8>(vbase, offA[j]);
-      offsets(min(ci + ws, last), offB);
+      for (; ci <= last; ci += ws) {
+        consume(
+            ci, kA, vc,
+            [&] {
+              offsets(min(ci + ws, last), offA);
 #pragma unroll
-      for (int j = 0; j < NL; ++j) kB[j] = load_kv_raw<KV8>(kbase, offB[j]);
-      consume(ci, kA, vc);
-      ci += ws;
-      if (ci > last) break;
+              for (int j = 0; j < NL; ++j) kA[j] = load_kv_raw<KV8>(kbase, offA[j]);
+            },
+            [&] {
 #pragma unroll
-      for (int j = 0; j < NL; ++j) vc[j] = load_kv_raw<KV8>(vbase, offB[j]);
-      offsets(min(ci + ws, last), offA);
+              for (int j = 0; j < NL; ++j) vc[j] = load_kv_raw<KV8>(vbase, offA[j]);
+            });
+      }
+    } else {
+      // Keys of the next chunk are in flight while the current one is folded in. The
+      // prefetch is unconditional -- at the last chunk it re-reads that chunk, which
+      // has just arrived -- so the compiler's waits for the values before each use
+      // leave the next chunk's keys outstanding (a conditional load would make them
+      // wait for everything).
+      auto none = [] {};
+      uint32_t offB[NL];
+      Raw kB[NL];
+      while (ci <= last) {
 #pragma unroll
-      for (int j = 0; j < NL; ++j) kA[j] = load_kv_raw<KV8>(kbase, offA[j]);
-      consume(ci, kB, vc);
-      ci += ws;
+        for (int j = 0; j < NL; ++j) vc[j] = load_kv_raw<KV8>(vbase, offA[j]);
+        offsets(min(ci + ws, last), offB);
+#pragma unroll
+        for (int j = 0; j < NL; ++j) kB[j] = load_kv_raw<KV8>(kbase, offB[j]);
+        consume(ci, kA, vc, none, none);
+        ci += ws;
+        if (ci > last) break;
+#pragma unroll
+        for (int j = 0; j < NL; ++j) vc[j] = load_kv_raw<KV8>(vbase, offB[j]);
+        offsets(min(ci + ws, last), offA);
+#pragma unroll
+        for (int j = 0; j < NL; ++j) kA[j] = load_kv_raw<KV8>(kbase, offA[j]);
+        consume(ci, kB, vc, none, none);
+        ci += ws;
+      }
     }
   }
   // Head mt's weight sum over the wave's 4 token groups (its lanes share m_h).
