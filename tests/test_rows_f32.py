@@ -70,6 +70,8 @@ def _planned(steps, heads: int, kv_heads: int, head_dim: int, block_size: int, l
     meta = hip_attention.plan(ForwardMode.MIXED, torch.tensor(s.rows, dtype=torch.int32, device="cuda:0"),
                               torch.tensor(s.lengths, dtype=torch.int32, device="cuda:0"),
                               torch.from_numpy(s.table.astype(np.int32)).cuda(), block_size)
+    # the tiles whatever the launch model prefers: it leaves short steps to the row kernel
+    meta.plan.splits[("row-tiles", kv_heads, heads // kv_heads, head_dim)] = True
     buffers = KVBuffers(_f32(s.k), _f32(s.v), KVLayoutKind.NHD if layout == "nhd" else KVLayoutKind.HND, RAW_CODEC)
     return s, meta, buffers, _f32(s.q)
 
@@ -81,7 +83,6 @@ def _planned(steps, heads: int, kv_heads: int, head_dim: int, block_size: int, l
 def test_row_tiles_match_the_oracle(heads: int, kv_heads: int, head_dim: int, block_size: int, layout: str) -> None:
     for n, steps in enumerate(STEPS):
         s, meta, buffers, q = _planned(steps, heads, kv_heads, head_dim, block_size, layout, 710 + n)
-        assert meta.plan.row_tiles(kv_heads, heads // kv_heads, head_dim), steps
         expected = s.expected(np.float64)
         out = torch.full_like(q, 7.0)
         for _ in range(2):  # recorded, then replayed
