@@ -251,9 +251,7 @@ class HipAttentionPlan:
         key = ("row-tiles", num_kv_heads, group, head_dim)
         found = self.splits.get(key)
         if found is None:
-            live = [count for count, length in zip(self.rows, self.kv_lengths) if count and length]
-            found = bool(live) and row_tiles_faster(live, self.max_length, sum(self.row_lengths), num_kv_heads, group,
-                                                    head_dim)
+            found = row_tiles_faster(self.rows, self.kv_lengths, num_kv_heads, group, head_dim)
             self.splits[key] = found
         return found
 
@@ -805,37 +803,79 @@ def prefill_model_us(group_lengths: list[int], row_lengths: tuple[int, ...] | li
     return t
 
 
-#: An fp32 step in tiles of rows (``paged_rows_f32_kernel``), modelled: a workgroup's fixed time, the
-#: time of one 16-position step of each of its waves by head width and 16-pair groups per tile, and
-#: the rate (flops per us) of a launch that fills the GPU. Row by row: a fixed time and the rate
-#: (bytes per us) at which every row streams its own context. Fitted to 60 steps (3 and 8 key/value
-#: heads, GQA 2 to 8, head widths 64 to 256, 2 to 2000 rows over 64 to 8192 positions), measured both
-#: ways: the faster side was taken on all but three, whose two sides are within 20%.
-ROW_TILES_FIXED_US = 6.0
-ROW_TILES_STEP_US = {(64, 1): 1.5, (64, 2): 3.0, (128, 1): 2.9, (128, 2): 3.6, (256, 1): 2.9}
-ROW_TILES_FLOPS_PER_US = 8.0e7
-ROWS_FIXED_US = 10.0
+#: An fp32 step in tiles of rows (``paged_rows_f32_kernel``), modelled, by head width and 16-pair
+#: groups per tile: the launch's fixed time, a workgroup's time per request that its tile walks (its
+#: table, the meeting of its waves, its output) and per 16-position step of each of its waves, in us.
+#: The workgroups run one per compute unit, and the contexts are streamed once (bytes per us).
+ROW_TILES_US = {(64, 1): (2.4, 2.7, 1.7), (64, 2): (4.9, 3.7, 2.7), (128, 1): (3.4, 4.2, 3.0),
+                (128, 2): (8.6, 5.0, 3.2), (256, 1): (2.9, 5.3, 4.2)}
+ROW_TILES_BYTES_PER_US = 5.5e6
+#: Row by row: a fixed time by head width, and the rate (bytes per us) at which every row streams its
+#: own context (rows of a request find most of it in the caches); with 8 query heads per wave half
+#: as much again of the one and three quarters of the other.
+ROWS_FIXED_US = {64: 10.0, 128: 18.0, 256: 20.0}
 ROWS_BYTES_PER_US = 8.0e6
-#: How much faster the tiles must model (their work depends more on how rows fall into tiles).
-ROW_TILES_MARGIN = 1.15
+ROWS_WIDE_FIXED, ROWS_WIDE_RATE = 1.5, 0.775
 
 
-def row_tiles_faster(rows: list[int], longest: int, total: int, num_kv_heads: int, group: int, head_dim: int) -> bool:
-    """Whether an fp32 multi-row step models faster in tiles of rows than row by row: ``rows`` the
-    rows of its requests with context, ``longest`` the longest context and ``total`` the sum of
-    its rows' contexts. A tile holds 16 or 32 consecutive (row, query head) pairs and walks its
-    requests one after the other, so short requests cost it their contexts in turn."""
-    pairs = sum(rows) * group
-    groups = 2 if head_dim != 256 and -(-pairs // 32) * num_kv_heads >= 2 * COMPUTE_UNITS else 1
-    waves = 4 if head_dim == 256 or (head_dim == 128 and groups == 2) else 8
-    tile, least = 16 * groups, min(rows) * group
-    aligned = all(count * group % tile == 0 for count in rows)
-    requests = min(len(rows), -(-tile // least) if aligned or least < tile and tile % least == 0
-                   else 1 + -(-(tile - 1) // least))
-    chain = requests * -(-longest // (16 * waves)) * ROW_TILES_STEP_US[(head_dim, groups)]
-    tiles = ROW_TILES_FIXED_US + max(chain, 4 * num_kv_heads * group * head_dim * total / ROW_TILES_FLOPS_PER_US)
-    by_row = ROWS_FIXED_US + total * num_kv_heads * 2 * head_dim * 4 / ROWS_BYTES_PER_US
-    return tiles * ROW_TILES_MARGIN < by_row
+def row_tile_shape(n_rows: int, num_kv_heads: int, group: int, head_dim: int) -> tuple[int, int]:
+    """(row, query head) pairs per tile and waves per workgroup of an fp32 step in tiles of rows
+    (mirrors ``rows_f32_groups`` and ``rows_f32_waves`` of the library: a test compares the tiles)."""
+    groups = 2 if head_dim != 256 and -(-n_rows * group // 32) * num_kv_heads >= 2 * COMPUTE_UNITS else 1
+    return 16 * groups, 4 if head_dim == 256 or (head_dim == 128 and groups == 2) else 8
+
+
+def row_tile_walks(rows: np.ndarray, lengths: np.ndarray, group: int, pairs: int,
+                   waves: int) -> tuple[np.ndarray, np.ndarray]:
+    """What each tile of ``pairs`` consecutive (row, query head) pairs walks: its requests, and the
+    16-position steps of its longest wave over all of them (a request's up to its last row of the
+    tile). Every request has rows; one of length 0 has no context."""
+    end = rows.cumsum() * group
+    start = end - rows * group
+    first = start // pairs
+    count = (end - 1) // pairs - first + 1  # tiles that hold rows of the request
+    request = np.arange(rows.size).repeat(count)
+    tile = np.arange(request.size) + (first - count.cumsum() + count)[request]
+    last_row = (np.minimum(tile * pairs + pairs, end[request]) - 1 - start[request]) // group
+    # the last of the row's positions, and with it the number of steps of the longest wave
+    steps = ((lengths - rows)[request] + last_row) // (16 * waves) + 1
+    steps[lengths[request] <= 0] = 0
+    return np.bincount(tile), np.bincount(tile, weights=steps)
+
+
+def row_tiles_faster(rows: "tuple[int, ...] | list[int]", lengths: "tuple[int, ...] | list[int]", num_kv_heads: int,
+                     group: int, head_dim: int) -> bool:
+    """Whether an fp32 multi-row step of ``rows`` query rows over contexts of ``lengths`` per request
+    models faster in tiles of rows than row by row.
+
+    A tile walks its requests one after the other, all of its columns spent on each, so requests of
+    few rows cost it their contexts in turn: 512 one-row requests of 128 positions (9/3 heads of 64)
+    take 55 us in tiles and 18 row by row, 64 requests of 4 rows over 1000 positions 36 and 76.
+    Fitted to 290 steps and checked on 710 more (1 to 600 requests of 1 to 2000 rows over up to 8192
+    positions, 1 to 32 key/value heads, GQA 1 to 8, every head width), each measured both ways: the
+    choice takes 1.6% more than the faster side on average; it takes tiles where row by row is more
+    than 5% faster on 10 of them (the worst: 376 requests of mostly one row, 32/32 heads of 64, 455
+    and 284 us).
+    """
+    counts = np.array(rows, dtype=np.int64)
+    contexts = np.array(lengths, dtype=np.int64)
+    if not counts.all():  # requests without rows hold no pairs
+        counts, contexts = counts[counts > 0], contexts[counts > 0]
+    seen = np.where(contexts > 0, counts, 0)  # rows with context
+    positions = int((seen * (2 * contexts - seen + 1)).sum()) // 2  # of all rows' contexts
+    if not positions:
+        return False
+    row_bytes = num_kv_heads * 2 * head_dim * 4
+    wide = group // head_chunks(group) == 8
+    by_row = (ROWS_FIXED_US[head_dim] * (ROWS_WIDE_FIXED if wide else 1.0)
+              + positions * row_bytes / (ROWS_BYTES_PER_US * (ROWS_WIDE_RATE if wide else 1.0)))
+    pairs, waves = row_tile_shape(int(counts.sum()), num_kv_heads, group, head_dim)
+    fixed, per_request, per_step = ROW_TILES_US[(head_dim, pairs // 16)]
+    requests, steps = row_tile_walks(counts, contexts, group, pairs, waves)
+    # a tile runs once per key/value head: that many workgroups of its length side by side
+    busy = _dispatch_makespan(per_request * requests + per_step * steps, max(1, COMPUTE_UNITS // num_kv_heads))
+    tiles = fixed + max(busy, int(contexts.sum()) * row_bytes / ROW_TILES_BYTES_PER_US)
+    return tiles < by_row
 
 
 def choose_prefill_partition(group_lengths: list[int], row_lengths: tuple[int, ...] | list[int],

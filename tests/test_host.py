@@ -368,6 +368,54 @@ def test_multi_row_launch_choice() -> None:
     assert pairs < 128 and size > 0
 
 
+def test_fp32_row_tiles_choice() -> None:
+    # (rows, contexts, heads, kv_heads, head_dim) and the times measured row by row and in tiles (us)
+    steps = [
+        (([1000], [1000]), (32, 8, 128), (500, 139)),  # a long prompt
+        (([362, 643], [362, 643]), (9, 3, 64), (42, 17)),  # two prompts
+        (([4] * 64, [1000] * 64), (9, 3, 64), (75.7, 35.8)),  # windows
+        (([8] * 60, [600] * 60), (16, 8, 256), (721, 112)),
+        (([256] + [1] * 30, [1000] + [500] * 30), (64, 8, 128), (335, 156)),  # a chunk beside decode rows
+        (([1] * 512, [128] * 512), (9, 3, 64), (18.1, 54.5)),  # one-row requests: a tile walks up to 11 of them
+        (([1] * 512, [1024] * 512), (32, 4, 64), (185, 229)),
+        (([1] * 256, [128] * 256), (32, 8, 64), (23.2, 39.0)),
+        (([1] * 512, [128] * 512), (32, 8, 128), (90.7, 177)),
+        (([1] * 512, [128] * 512), (64, 8, 128), (110, 182)),
+        (([1] * 512, [128] * 512), (16, 8, 256), (169, 216)),
+        (([1] * 256, [128] * 256), (16, 16, 64), (41.8, 73.9)),
+        (([1] * 16, [4096] * 16), (8, 8, 128), (84, 1595)),
+        (([2] * 4, [1000] * 4), (9, 3, 64), (11.8, 44.1)),  # few rows: too few workgroups
+        (([24] * 40, [24] * 40), (32, 8, 64), (25.1, 37.3)),  # many short prompts
+    ]
+    for (rows, lengths), (heads, kv_heads, head_dim), (row_us, tile_us) in steps:
+        got = hip_attention.row_tiles_faster(rows, lengths, kv_heads, heads // kv_heads, head_dim)
+        assert got == (tile_us < row_us), (rows[:3], lengths[:3], heads, kv_heads, head_dim)
+    # requests without rows change nothing; padding requests hold pairs but no context
+    assert hip_attention.row_tiles_faster([0, 1000, 0], [50, 1000, 0], 8, 4, 128)
+    assert hip_attention.row_tiles_faster([1000, 2], [1000, 0], 8, 4, 128)
+    assert not hip_attention.row_tiles_faster([3, 2], [0, 0], 8, 4, 128)
+    assert not hip_attention.row_tiles_faster([], [], 8, 4, 128)
+
+
+def test_fp32_row_tiles_walk_their_requests_one_by_one() -> None:
+    rng = np.random.default_rng(91)
+    for case in range(60):
+        group, pairs, waves = int(rng.integers(1, 21)), int(rng.choice([16, 32])), int(rng.choice([1, 4, 8]))
+        rows = rng.integers(1, [3, 9, 80][case % 3], size=int(rng.integers(1, 30)))
+        lengths = np.where(rng.random(rows.size) < 0.1, 0, rows + rng.integers(0, 500, size=rows.size))
+        owner = np.repeat(np.arange(rows.size), rows * group)  # of each pair
+        row = np.concatenate([np.repeat(np.arange(n), group) for n in rows])
+        requests, steps = [], []
+        for at in range(0, owner.size, pairs):
+            longest: dict[int, int] = {}
+            for r, j in zip(owner[at:at + pairs], row[at:at + pairs]):
+                longest[r] = int(lengths[r] - rows[r] + j + 1) if lengths[r] else 0
+            requests.append(len(longest))
+            steps.append(sum(-(-n // (16 * waves)) for n in longest.values()))
+        got = hip_attention.row_tile_walks(rows, lengths, group, pairs, waves)
+        assert got[0].tolist() == requests and got[1].tolist() == steps, case
+
+
 def test_multi_row_launch_choice_by_head_width() -> None:
     def launch(rows: list[int], lengths: list[int], heads: int, head_dim: int, kv_heads: int = 8) -> tuple[int, int]:
         table = torch.ones(len(rows), max(lengths) // 16 + 1, dtype=torch.int32)

@@ -48,6 +48,53 @@ def test_row_tiles_read_inside_the_cache(head_dim: int) -> None:
         reach._check(step, got, f"row tiles case {case} bs {bs}")
 
 
+def test_the_modelled_tiles_are_the_launched_ones() -> None:
+    # the launch model and the library agree on the pairs of a tile: every load of the launch is one of a
+    # step that the model counts (16 positions: head_dim / 16 key and head_dim / 16 value loads per lane)
+    rng = np.random.default_rng(705)
+    for case in range(24):
+        head_dim = (64, 128, 256)[case % 3]
+        kv_heads, group = [(8, 4), (3, 3), (1, 20), (8, 8), (16, 1)][case % 5]
+        lengths = [int(n) for n in rng.integers(1, 200, size=int(rng.integers(1, 60)))]
+        step = reach.Step(rng, lengths, 16, kv_heads, head_dim, False, case % 2, fp32=True)
+        rows = [max(1, n // (1, 2, 20)[case % 3]) for n in lengths]
+        req, pos = reach._rows(step, rows)
+        args = reach._common(step, kv_heads * group, len(req), req, pos)
+        loads = int(reach._walk(step, lambda lib: lib.ayk_paged_attention_v1(*args, hip_attention.ROW_TILES, None))[2])
+        pairs, _ = hip_attention.row_tile_shape(len(req), kv_heads, group, head_dim)
+        steps = hip_attention.row_tile_walks(np.array(rows), np.array(lengths), group, pairs, 1)[1].sum()
+        assert loads == steps * kv_heads * 64 * head_dim // 8, (case, pairs)
+    # two groups from 2 x 256 workgroups of 32 pairs: 504 and 505 rows make 63 and 64 tiles x 8 heads
+    assert hip_attention.row_tile_shape(504, 8, 4, 64)[0] == 16 and hip_attention.row_tile_shape(505, 8, 4, 64)[0] == 32
+
+
+def test_attend_runs_the_launch_that_the_model_picks(monkeypatch: pytest.MonkeyPatch) -> None:
+    # with the address walk on nothing launches, so the recorded call can be looked at on the CPU
+    monkeypatch.setattr(hip_attention, "stream_handle", lambda device: 0)
+    monkeypatch.setattr(hip_attention, "require_buffers", lambda op, buffers: None)
+    monkeypatch.setattr(hip_attention, "_workspace", lambda *a: torch.zeros(1 << 24, dtype=torch.uint8))
+    monkeypatch.setattr(hip_attention, "_arrivals", lambda *a: torch.zeros(1 << 12, dtype=torch.int32))
+    lib = _lib.lib()
+
+    def call(rows: list[int], lengths: list[int], mode: ForwardMode) -> tuple[str, int]:
+        s = build_scenario(list(zip(rows, lengths)), heads=9, kv_heads=3, head_dim=64, block_size=16, mode=mode.value)
+        meta = hip_attention.plan(mode, torch.tensor(rows), torch.tensor(lengths), torch.from_numpy(s.table), 16)
+        q = torch.zeros(sum(rows), 9, 64)
+        buffers = KVBuffers(torch.zeros(s.k.shape), torch.zeros(s.k.shape), KVLayoutKind.NHD, RAW_CODEC)
+        assert lib.ayk_debug_kv_reach_begin(s.table.size) == 0
+        try:
+            hip_attention.attend(q, buffers, meta, torch.zeros_like(q), scale=0.125)
+        finally:
+            assert lib.ayk_debug_kv_reach_end(np.zeros(5, dtype=np.int64).ctypes.data) == 0
+        (found,) = meta.plan.launches.values()
+        return found.fn.__name__, found.args[-1].value
+
+    assert call([300, 200], [300, 500], ForwardMode.MIXED) == ("ayk_paged_attention_v1", hip_attention.ROW_TILES)
+    for rows, mode in (([1] * 40, ForwardMode.MIXED), ([1] * 40, ForwardMode.DECODE)):
+        name, flags = call(rows, [200] * 40, mode)
+        assert not flags & hip_attention.ROW_TILES, (name, mode)
+
+
 def test_row_tiles_are_refused_elsewhere() -> None:
     lib = _lib.lib()
 
