@@ -48,6 +48,21 @@ def test_row_tiles_read_inside_the_cache(head_dim: int) -> None:
         reach._check(step, got, f"row tiles case {case} bs {bs}")
 
 
+@pytest.mark.parametrize("head_dim", [64, 128])
+def test_two_group_row_tiles_read_inside_the_cache(head_dim: int) -> None:
+    rng = np.random.default_rng(706 + head_dim)
+    for case, bs in enumerate(reach.BLOCK_SIZES):
+        kv_heads, group = [(8, 4), (8, 3), (8, 5), (24, 1)][case % 4]
+        rows = [532, 19, 26, 140]
+        lengths = [600, 200, 26, -(-300 // bs) * bs]
+        step = reach.Step(rng, lengths, bs, kv_heads, head_dim, False, case % 2, fp32=True)
+        req, pos = reach._rows(step, rows)
+        assert hip_attention.row_tile_shape(len(req), kv_heads, group, head_dim)[0] == 32
+        args = reach._common(step, kv_heads * group, len(req), req, pos)
+        got = reach._walk(step, lambda lib: lib.ayk_paged_attention_v1(*args, hip_attention.ROW_TILES, None))
+        reach._check(step, got, f"two-group row tiles case {case} bs {bs}")
+
+
 def test_the_modelled_tiles_are_the_launched_ones() -> None:
     # the launch model and the library agree on the pairs of a tile: every load of the launch is one of a
     # step that the model counts (16 positions: head_dim / 16 key and head_dim / 16 value loads per lane)
@@ -123,31 +138,52 @@ def _planned(steps, heads: int, kv_heads: int, head_dim: int, block_size: int, l
     return s, meta, buffers, _f32(s.q)
 
 
+def _assert_matches(steps, heads: int, kv_heads: int, head_dim: int, block_size: int, layout: str,
+                    seed: int) -> None:
+    s, meta, buffers, q = _planned(steps, heads, kv_heads, head_dim, block_size, layout, seed)
+    expected = s.expected(np.float64)
+    out = torch.full_like(q, 7.0)
+    for _ in range(2):  # recorded, then replayed
+        hip_attention.attend(q, buffers, meta, out, scale=s.scale)
+    torch.cuda.synchronize()
+    got = out.double().cpu().numpy()
+    bound = 4 * EPS32 * float(np.abs(expected).max()) + 1e-6
+    assert np.isfinite(got).all(), steps
+    assert float(np.abs(got - expected).max()) <= bound, steps
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("heads,kv_heads,head_dim", [(9, 3, 64), (32, 8, 64), (8, 2, 128), (5, 5, 128), (20, 1, 128),
                                                      (16, 8, 256), (6, 2, 256)])
 @pytest.mark.parametrize("block_size,layout", [(16, "nhd"), (24, "hnd"), (5, "nhd"), (1, "hnd")])
 def test_row_tiles_match_the_oracle(heads: int, kv_heads: int, head_dim: int, block_size: int, layout: str) -> None:
     for n, steps in enumerate(STEPS):
-        s, meta, buffers, q = _planned(steps, heads, kv_heads, head_dim, block_size, layout, 710 + n)
-        expected = s.expected(np.float64)
-        out = torch.full_like(q, 7.0)
-        for _ in range(2):  # recorded, then replayed
-            hip_attention.attend(q, buffers, meta, out, scale=s.scale)
-        torch.cuda.synchronize()
-        got = out.double().cpu().numpy()
-        bound = 4 * EPS32 * float(np.abs(expected).max()) + 1e-6
-        assert np.isfinite(got).all(), steps
-        assert float(np.abs(got - expected).max()) <= bound, steps
+        _assert_matches(steps, heads, kv_heads, head_dim, block_size, layout, 710 + n)
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("head_dim", [64, 256])
-def test_values_that_are_not_finite_reach_only_the_rows_that_see_them(head_dim: int) -> None:
-    s, meta, buffers, q = _planned([(40, 70)], 8, 2, head_dim, 16, "nhd", 720)
+@pytest.mark.parametrize("heads,kv_heads,head_dim,block_size,layout",
+                         [(32, 8, 64, 16, "nhd"), (24, 8, 64, 5, "hnd"), (32, 8, 128, 24, "hnd"), (40, 8, 128, 16, "nhd")])
+def test_two_group_row_tiles_match_the_oracle(heads: int, kv_heads: int, head_dim: int, block_size: int,
+                                              layout: str) -> None:
+    # a border between a tile's two 16-pair groups (532 rows of 4 heads), tiles that hold two requests'
+    # rows and padding rows, a ragged last tile
+    steps = [(532, 560), (9, 0), (19, 200), (26, 26), (100, 250)]
+    rows = sum(count for count, _ in steps)
+    assert hip_attention.row_tile_shape(rows, kv_heads, heads // kv_heads, head_dim)[0] == 32
+    _assert_matches(steps, heads, kv_heads, head_dim, block_size, layout, 730)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("head_dim,steps,pairs", [(64, [(40, 70)], 16), (256, [(40, 70)], 16), (64, [(600, 630)], 32),
+                                                  (128, [(600, 630)], 32)])
+def test_values_that_are_not_finite_reach_only_the_rows_that_see_them(head_dim: int, steps, pairs: int) -> None:
+    heads, kv_heads = (32, 8) if pairs == 32 else (8, 2)
+    assert hip_attention.row_tile_shape(steps[0][0], kv_heads, 4, head_dim)[0] == pairs
+    s, meta, buffers, q = _planned(steps, heads, kv_heads, head_dim, 16, "nhd", 720)
     clean, out = torch.empty_like(q), torch.empty_like(q)
     hip_attention.attend(q, buffers, meta, clean, scale=s.scale)
-    at = 53  # positions 30 to 69 are the rows; rows before position 53 do not see it
+    at = 53  # the rows are positions 30 up; rows before position 53 do not see it
     block, offset = int(s.table[0][at // 16]), at % 16
     buffers.v[block, offset, 0, 3] = float("inf")
     buffers.v[block, offset, 1, 5] = float("nan")
@@ -158,8 +194,9 @@ def test_values_that_are_not_finite_reach_only_the_rows_that_see_them(head_dim: 
     # the contract's bound on each side of the exact result
     bound = 2 * (4 * EPS32 * float(clean.abs().max()) + 1e-6)
     assert float((out[:before] - clean[:before]).abs().nan_to_num(float("inf")).max()) <= bound
-    assert torch.isinf(out[before:, :4, 3]).all() and torch.isnan(out[before:, 4:, 5]).all()
+    assert torch.isinf(out[before:, :4, 3]).all() and torch.isnan(out[before:, 4:8, 5]).all()
     kept = torch.ones(head_dim, dtype=torch.bool, device="cuda:0")
     kept[3] = False
     others = (out[before:, :4] - clean[before:, :4])[:, :, kept]
     assert float(others.abs().nan_to_num(float("inf")).max()) <= bound
+    assert torch.equal(out[:, 8:], clean[:, 8:])
