@@ -19,6 +19,8 @@ from ayaka_amd.enums import ForwardMode, KVLayoutKind
 from ayaka_amd.hip import _lib
 from ayaka_amd.hip import attention as hip_attention
 from ayaka_amd.kvcache import RAW_CODEC, KVBuffers
+from oracle import paged
+from oracle.numerics import bits_to_f32, f32_to_bits
 from tests import test_kv_reach as reach
 from tests._support import build_scenario
 
@@ -126,22 +128,35 @@ def _f32(a: np.ndarray) -> torch.Tensor:
     return torch.from_numpy(np.ascontiguousarray(a, dtype=np.float32)).to("cuda:0")
 
 
+def _full_mantissas(like: np.ndarray, rng: np.random.Generator) -> np.ndarray:
+    """float32 normals with all their bits where ``like`` (values of a 16-bit type) is not NaN, so that an
+    operand shortened on its way to the products shows: bf16 would move a value by up to 2^-9 of it."""
+    fresh = rng.standard_normal(like.shape).astype(np.float32)
+    assert np.mean(fresh != bits_to_f32(f32_to_bits(fresh, "bf16"), "bf16")) > 0.99
+    return np.where(np.isnan(like), like, fresh)
+
+
 def _planned(steps, heads: int, kv_heads: int, head_dim: int, block_size: int, layout: str, seed: int):
+    """A planned step in tiles, its caches and queries on the GPU, and the oracle's float64 output."""
     s = build_scenario(steps, heads=heads, kv_heads=kv_heads, head_dim=head_dim, block_size=block_size,
                        layout=layout, mode="mixed", seed=seed)
+    rng = np.random.default_rng(seed + 1000)
+    q, k, v = (_full_mantissas(a, rng) for a in (s.q, s.k, s.v))
     meta = hip_attention.plan(ForwardMode.MIXED, torch.tensor(s.rows, dtype=torch.int32, device="cuda:0"),
                               torch.tensor(s.lengths, dtype=torch.int32, device="cuda:0"),
                               torch.from_numpy(s.table.astype(np.int32)).cuda(), block_size)
     # the tiles whatever the launch model prefers: it leaves short steps to the row kernel
     meta.plan.splits[("row-tiles", kv_heads, heads // kv_heads, head_dim)] = True
-    buffers = KVBuffers(_f32(s.k), _f32(s.v), KVLayoutKind.NHD if layout == "nhd" else KVLayoutKind.HND, RAW_CODEC)
-    return s, meta, buffers, _f32(s.q)
+    buffers = KVBuffers(_f32(k), _f32(v), KVLayoutKind.NHD if layout == "nhd" else KVLayoutKind.HND, RAW_CODEC)
+    expected = paged.attention(q, k, v, s.table, np.asarray(s.lengths), scale=s.scale, layout=layout,
+                               request_of_row=s.plan["request_of_row"], positions=s.plan["positions"],
+                               precision=np.float64)
+    return s, meta, buffers, _f32(q), expected
 
 
 def _assert_matches(steps, heads: int, kv_heads: int, head_dim: int, block_size: int, layout: str,
                     seed: int) -> None:
-    s, meta, buffers, q = _planned(steps, heads, kv_heads, head_dim, block_size, layout, seed)
-    expected = s.expected(np.float64)
+    s, meta, buffers, q, expected = _planned(steps, heads, kv_heads, head_dim, block_size, layout, seed)
     out = torch.full_like(q, 7.0)
     for _ in range(2):  # recorded, then replayed
         hip_attention.attend(q, buffers, meta, out, scale=s.scale)
@@ -180,7 +195,7 @@ def test_two_group_row_tiles_match_the_oracle(heads: int, kv_heads: int, head_di
 def test_values_that_are_not_finite_reach_only_the_rows_that_see_them(head_dim: int, steps, pairs: int) -> None:
     heads, kv_heads = (32, 8) if pairs == 32 else (8, 2)
     assert hip_attention.row_tile_shape(steps[0][0], kv_heads, 4, head_dim)[0] == pairs
-    s, meta, buffers, q = _planned(steps, heads, kv_heads, head_dim, 16, "nhd", 720)
+    s, meta, buffers, q, _ = _planned(steps, heads, kv_heads, head_dim, 16, "nhd", 720)
     clean, out = torch.empty_like(q), torch.empty_like(q)
     hip_attention.attend(q, buffers, meta, clean, scale=s.scale)
     at = 53  # the rows are positions 30 up; rows before position 53 do not see it
