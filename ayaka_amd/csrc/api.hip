@@ -215,8 +215,9 @@ int wave_split_for(const ayk::AttnParams& p, bool split, int32_t flags) {
 }
 
 // The q.k path and workgroup shape for a launch, then the kernel(s).
-// fp32 models: the VALU decode kernel, one wave per virtual head, partitions merged by its own
-// reduce kernel (no wave split, no single launch, no q.k choice).
+// fp32 models: tiles of rows on the matrix cores where the caller asks for them (v1 over rows with
+// positions), else the VALU decode kernel, each row on its own: one wave per virtual head,
+// partitions merged by its own reduce kernel (no wave split, no single launch, no q.k choice).
 int launch_f32(const char* op, const ayk::AttnParams& p, int head_dim, int gc, bool split, int32_t flags,
                void* stream) {
   if (!split && flags == AYK_FLAG_ROW_TILES && p.positions) {
@@ -229,9 +230,8 @@ int launch_f32(const char* op, const ayk::AttnParams& p, int head_dim, int gc, b
     return launched(ayk::launch_rows_f32(p, head_dim, compute_units(), static_cast<hipStream_t>(stream)), op);
   }
   if (flags & ~(AYK_FLAG_PARTIALS_ONLY | AYK_FLAG_SEPARATE_REDUCE | AYK_FLAG_WAVES_1))
-    return fail(AYK_ERR_UNSUPPORTED, "%s: flags 0x%x: fp32 runs one kernel shape (partials only, a separate "
-                "reduce and one wave per head are the flags it takes; v1 also row tiles alone, over rows with "
-                "positions)", op, flags);
+    return fail(AYK_ERR_UNSUPPORTED, "%s: flags 0x%x: fp32 takes partials only, a separate reduce and one wave "
+                "per head, or, in v1 over rows with positions, row tiles alone", op, flags);
   ayk::AttnParams q = p;
   q.wave_split = 1;
   q.arrivals = nullptr;
@@ -545,7 +545,7 @@ int ayk_paged_prefill(void* out, const void* q, const void* k_cache, const void*
   const int rc = prepare(op, c, p, gc);
   if (rc != AYK_OK) return rc;
   if (dtype == AYK_DTYPE_FP32)
-    return fail(AYK_ERR_UNSUPPORTED, "%s: fp32 runs on the decode entry points, row by row", op);
+    return fail(AYK_ERR_UNSUPPORTED, "%s: fp32 runs on the decode entry points (multi-row steps too)", op);
   // Tiles of the full capacity, or of a half or a quarter (2 or 4 waves then share
   // each group of pairs and split its chunks), or at head_dim 128 and 256 of twice it (an
   // 8-wave workgroup; waves_per_group 0 below).
@@ -632,7 +632,7 @@ int ayk_paged_attention_windows(void* out, const void* q, const void* k_cache, c
   const int rc = prepare(op, c, p, gc);
   if (rc != AYK_OK) return rc;
   if (dtype == AYK_DTYPE_FP32)
-    return fail(AYK_ERR_UNSUPPORTED, "%s: fp32 runs on the decode entry points, row by row", op);
+    return fail(AYK_ERR_UNSUPPORTED, "%s: fp32 runs on the decode entry points (multi-row steps too)", op);
   if (p.group > 16)
     return fail(AYK_ERR_UNSUPPORTED, "%s: %d query heads per key/value head exceed a window's 16 columns", op,
                 p.group);

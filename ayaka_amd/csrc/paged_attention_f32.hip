@@ -4,8 +4,8 @@
 // over fp32 caches, which its torch backend serves and flashinfer refuses
 // (python/ayaka/ops/backends/flashinfer/attention.py:298-301): row n attends to positions
 // [0, len_n) of its request, scores scale * q.k, softmax and the value sum in fp32, and the
-// output written in fp32. Rows with a position (multi-row steps run row by row here) see
-// [0, position].
+// output written in fp32. Rows with a position (those of multi-row steps that run row by row,
+// not in the tiles of paged_rows_f32_kernel) see [0, position].
 //
 // The path is bandwidth-bound like the 16-bit decode kernels, with twice the bytes per
 // position, so it keeps their shape on the VALU: one workgroup per (row[, partition]) and group

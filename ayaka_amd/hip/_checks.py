@@ -2,8 +2,8 @@
 
 The messages follow the reference's (``python/ayaka/ops/backends/torch/_checks.py:21-59``,
 ``kvcache.py:39-62``) so that callers and tests read the same refusals. The
-hip backend computes in fp16, bf16 and fp32 (fp32 on a decode kernel of its own, row by row),
-on HIP devices, for head widths of 64, 128 and 256 and block sizes of 1 to 65536 positions; it
+hip backend computes in fp16, bf16 and fp32 (fp32 on kernels of its own: one for decode and for rows
+one by one, one for tiles of rows), on HIP devices, for head widths of 64, 128 and 256 and block sizes of 1 to 65536 positions; it
 stores the ``"raw"`` codec (fp16/bf16/fp32 caches) and ``"fp8_e4m3"`` (``float8_e4m3fn`` caches,
 read by fp16/bf16 models).
 """
@@ -32,7 +32,7 @@ __all__ = [
 
 HEAD_DIMS = frozenset({64, 128, 256})
 _DTYPES = (torch.float16, torch.bfloat16)  # compute dtypes over a quantised codec
-_RAW_DTYPES = (torch.float16, torch.bfloat16, torch.float32)  # the raw codec's, fp32 on its own kernel
+_RAW_DTYPES = (torch.float16, torch.bfloat16, torch.float32)  # the raw codec's, fp32 on its own kernels
 _NAMES = {
     torch.float16: "float16",
     torch.bfloat16: "bfloat16",

@@ -1118,8 +1118,8 @@ def attend_with(
                      and not partials_only and merge is None and waves is None
                      and step.row_tiles(kv_heads, heads // kv_heads, buffers.head_dim))
         if prefill or window or (qk is not None) or (waves not in (None, 1)) or merge == "in-kernel":
-            raise BackendError(f"{op}: fp32 runs one launch shape: the per-row decode kernel, one wave per "
-                               "head, partitions merged by the reduce kernel", context={"op": op})
+            raise BackendError(f"{op}: fp32 runs one launch shape that can be forced: the per-row decode kernel, "
+                               "one wave per head, partitions merged by the reduce kernel", context={"op": op})
         prefill = False
     if prefill is None:
         prefill = not decode and _wants_prefill_kernel(step)

@@ -1,10 +1,11 @@
-"""fp32 models on the hip backend: the fp32 decode kernel against the float64 oracle.
+"""fp32 models on the hip backend: the fp32 kernels against the float64 oracle.
 
 The reference's torch backend serves fp32 (``python/ayaka/ops/backends/torch/_checks.py:30-38``);
 its contract tests hold fp32 outputs to ``4 * eps * max|y| + 1e-6`` against float64
 (``tests/ops/test_attention_contract.py:168-171``), the bound used here. Decode steps run v1
 and v2 (either grid, partitions merged by the fp32 reduce kernel); multi-row steps run row by
-row on the same kernel; graph replays read their staged split.
+row on the same kernel where the launch is forced, and as the launch model picks (row by row or in
+tiles of rows) where it is not; graph replays read their staged split.
 """
 
 from __future__ import annotations

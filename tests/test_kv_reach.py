@@ -247,7 +247,7 @@ def test_the_walk_reports_out_of_range_tables() -> None:
 @pytest.mark.parametrize("head_dim", [64, 128, 256])
 def test_fp32_decode_loads_stay_in_the_cache(head_dim: int) -> None:
     # the fp32 kernel: 16-byte loads of 4 floats, D / 4 lanes per position, v1 and v2 over every
-    # grid kind; multi-row steps of an fp32 model run row by row on it (rows carry positions)
+    # grid kind; multi-row steps of an fp32 model that run row by row do so on it (rows carry positions)
     rng = np.random.default_rng(300 + head_dim)
     for case in range(20):
         bs = BLOCK_SIZES[case % len(BLOCK_SIZES)]
