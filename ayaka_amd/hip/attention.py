@@ -816,6 +816,9 @@ ROW_TILES_BYTES_PER_US = 5.5e6
 ROWS_FIXED_US = {64: 10.0, 128: 18.0, 256: 20.0}
 ROWS_BYTES_PER_US = 8.0e6
 ROWS_WIDE_FIXED, ROWS_WIDE_RATE = 1.5, 0.775
+#: The tiles are taken up to this ratio of the modelled times: the median of tiles modelled over tiles
+#: measured is 1.11 (950 steps; a ratio of 1 costs 2.4% over the faster side on them, 1.1 1.8%).
+ROW_TILES_MARGIN = 1.1
 
 
 def row_tile_shape(n_rows: int, num_kv_heads: int, group: int, head_dim: int) -> tuple[int, int]:
@@ -825,21 +828,31 @@ def row_tile_shape(n_rows: int, num_kv_heads: int, group: int, head_dim: int) ->
     return 16 * groups, 4 if head_dim == 256 or (head_dim == 128 and groups == 2) else 8
 
 
+def _row_tile_steps(rows: np.ndarray, lengths: np.ndarray, group: int, pairs: int,
+                    waves: int) -> tuple[np.ndarray, np.ndarray]:
+    """Per request and tile that holds rows of it: the tile, and the 16-position steps of the tile's
+    longest wave over the request (none without context). Every request has rows."""
+    owned = rows * group
+    end = owned.cumsum()
+    start = end - owned
+    first = start // pairs
+    count = (end - 1) // pairs + 1 - first
+    # the requests' tiles follow each other, a tile that two requests share once for each
+    tile = np.arange(count.sum()) - (count.cumsum() - count - first).repeat(count)
+    # the row's position of the request's last pair in the tile, in steps of the waves together
+    last = np.minimum((tile + 1) * pairs, end.repeat(count)) - 1 - start.repeat(count)
+    steps = ((lengths - rows).repeat(count) + last // group) // (16 * waves) + 1
+    if not lengths.all():
+        steps *= lengths.repeat(count) > 0
+    return tile, steps
+
+
 def row_tile_walks(rows: np.ndarray, lengths: np.ndarray, group: int, pairs: int,
                    waves: int) -> tuple[np.ndarray, np.ndarray]:
     """What each tile of ``pairs`` consecutive (row, query head) pairs walks: its requests, and the
     16-position steps of its longest wave over all of them (a request's up to its last row of the
     tile). Every request has rows; one of length 0 has no context."""
-    end = rows.cumsum() * group
-    start = end - rows * group
-    first = start // pairs
-    count = (end - 1) // pairs - first + 1  # tiles that hold rows of the request
-    request = np.arange(rows.size).repeat(count)
-    tile = np.arange(request.size) + (first - count.cumsum() + count)[request]
-    last_row = (np.minimum(tile * pairs + pairs, end[request]) - 1 - start[request]) // group
-    # the last of the row's positions, and with it the number of steps of the longest wave
-    steps = ((lengths - rows)[request] + last_row) // (16 * waves) + 1
-    steps[lengths[request] <= 0] = 0
+    tile, steps = _row_tile_steps(rows, lengths, group, pairs, waves)
     return np.bincount(tile), np.bincount(tile, weights=steps)
 
 
@@ -851,18 +864,20 @@ def row_tiles_faster(rows: "tuple[int, ...] | list[int]", lengths: "tuple[int, .
     A tile walks its requests one after the other, all of its columns spent on each, so requests of
     few rows cost it their contexts in turn: 512 one-row requests of 128 positions (9/3 heads of 64)
     take 55 us in tiles and 18 row by row, 64 requests of 4 rows over 1000 positions 36 and 76.
-    Fitted to 290 steps and checked on 710 more (1 to 600 requests of 1 to 2000 rows over up to 8192
-    positions, 1 to 32 key/value heads, GQA 1 to 8, every head width), each measured both ways: the
-    choice takes 1.6% more than the faster side on average; it takes tiles where row by row is more
-    than 5% faster on 10 of them (the worst: 376 requests of mostly one row, 32/32 heads of 64, 455
-    and 284 us).
+    Fitted to 290 steps (1 to 600 requests of 1 to 2000 rows over up to 8192 positions, 1 to 32
+    key/value heads, GQA 1 to 8, every head width) and checked on 950 others, each measured both
+    ways: 500 prompts, chunks, windows and mixed steps of the usual head shapes, on which the choice
+    takes 0.9% more than the faster side on average, and 450 of many short requests, 2.7%. It takes
+    tiles where row by row is more than 5% faster on 21 of them (the worst: 251 requests of 3 rows,
+    64/32 heads of 64, 177 and 121 us), and rows where tiles are on 44 (the worst: one key/value
+    head, whose rows it under-prices: 226 rows, 8 heads of 128, 160 and 70 us).
     """
     counts = np.array(rows, dtype=np.int64)
     contexts = np.array(lengths, dtype=np.int64)
     if not counts.all():  # requests without rows hold no pairs
         counts, contexts = counts[counts > 0], contexts[counts > 0]
-    seen = np.where(contexts > 0, counts, 0)  # rows with context
-    positions = int((seen * (2 * contexts - seen + 1)).sum()) // 2  # of all rows' contexts
+    seen = counts if contexts.all() else counts * (contexts > 0)  # rows with context
+    positions = int(seen.dot(2 * contexts - seen + 1)) // 2  # of all rows' contexts
     if not positions:
         return False
     row_bytes = num_kv_heads * 2 * head_dim * 4
@@ -871,11 +886,12 @@ def row_tiles_faster(rows: "tuple[int, ...] | list[int]", lengths: "tuple[int, .
               + positions * row_bytes / (ROWS_BYTES_PER_US * (ROWS_WIDE_RATE if wide else 1.0)))
     pairs, waves = row_tile_shape(int(counts.sum()), num_kv_heads, group, head_dim)
     fixed, per_request, per_step = ROW_TILES_US[(head_dim, pairs // 16)]
-    requests, steps = row_tile_walks(counts, contexts, group, pairs, waves)
+    tile, steps = _row_tile_steps(counts, contexts, group, pairs, waves)
     # a tile runs once per key/value head: that many workgroups of its length side by side
-    busy = _dispatch_makespan(per_request * requests + per_step * steps, max(1, COMPUTE_UNITS // num_kv_heads))
+    busy = _dispatch_makespan(np.bincount(tile, weights=per_step * steps + per_request),
+                              max(1, COMPUTE_UNITS // num_kv_heads))
     tiles = fixed + max(busy, int(contexts.sum()) * row_bytes / ROW_TILES_BYTES_PER_US)
-    return tiles < by_row
+    return tiles < by_row * ROW_TILES_MARGIN
 
 
 def choose_prefill_partition(group_lengths: list[int], row_lengths: tuple[int, ...] | list[int],
