@@ -312,8 +312,8 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void paged_attention_mfma_kernel
       // chunk's are in LDS (at the last chunk: that chunk again). With the two key buffers
       // below this width took 54-113 registers more than two waves per SIMD have, and the
       // spills bounded every chunk: 16/8 heads, us, before -> now: 32 rows of 4000 positions
-      // 241 -> 165 (6.4 TB/s), over fp8 caches 120 -> 87; 1 row of 500 28 -> 18; 4-row windows
-      // over 64 contexts of 1500 202 -> 124.
+      // 238 -> 163 (6.4 TB/s), over fp8 caches 123 -> 88; 1 row of 500 36 -> 20; 4-row windows
+      // over 64 contexts of 1500 201 -> 124.
 #pragma unroll
       for (int j = 0; j < NL; ++j) vc[j] = load_kv_raw<KV8>(vbase, offA[j]);
       for (; ci <= last; ci += ws) {

@@ -8,16 +8,19 @@
 // Row by row (paged_attention_f32_kernel) a prompt of n rows reads its context n times and runs
 // four FMAs per lane, key and head on the VALU. Here a workgroup serves one key/value head and a
 // tile of PT x 16 (row, query head) pairs, consecutive in the order (row, head of the group); the
-// tile's rows are walked request by request (one, or two where it spans a border), each wave
-// taking every W-th 16-position step of the context, and the waves' states meet in LDS in wave
-// order. Both contractions are v_mfma_f32_16x16x4f32 (fp32 products and sums), so nothing is
-// rounded to a shorter type. What bounds it: that instruction's rate (64 flops a cycle and SIMD,
-// 157 TFLOP/s; a large fp32 product reaches 150 here) on large steps, the chain of each wave's
-// steps (1.5 us per 16 positions at head_dim 64, 2.9 at 128) on small ones.
+// tile's rows are walked request by request, each wave taking every W-th 16-position step of the
+// context, and the waves' states meet in LDS in wave order. Both contractions are
+// v_mfma_f32_16x16x4f32 (fp32 products and sums), so nothing is rounded to a shorter type. What
+// bounds it: the chain of each wave's steps. A step of 16 positions takes 1.6 us at head_dim 64,
+// 2.8 at 128 and 3.3 at 256 with 16 pairs, 2.6 and 3.1 with 32, of which the products' own rate
+// (64 flops a cycle and SIMD, 157 TFLOP/s; a large fp32 product reaches 150 here) is about half at
+// 64 with 16 pairs; large steps reach 54-65 TFLOP/s. A tile of prompts spans one request or two, but
+// one of one-row requests up to 16 PT, each with its own pass over all columns, two barriers and a
+// merge (3-5 us): such steps are left to the row kernel by the caller's launch model.
 //
-// Measured, us, row by row -> here: 2 prompts of 450 rows, 9/3 heads of 64, 42 -> 17; 32/8 heads
-// of 64, one chunk of 300 rows over 3000 positions, 360 -> 111 (63 TFLOP/s), 1000-row prompt
-// 214 -> 72; 32/8 heads of 128, the same prompt, 503 -> 139; 16/8 heads of 256, 963 -> 145.
+// Measured, us, row by row -> here: 2 prompts of 592 and 491 rows, 9/3 heads of 64, 54 -> 23; 32/8
+// heads of 64, one chunk of 300 rows over 3000 positions, 364 -> 108 (65 TFLOP/s), 1000-row prompt
+// 225 -> 71; 32/8 heads of 128, the same prompt, 504 -> 134; 16/8 heads of 256, 980 -> 152.
 //
 //  * No operand goes through LDS. S^T = K Q^T: the contraction index is free to permute, so lane
 //    (mt, mq) of the key operand loads 16 contiguous bytes of position mt (dims 16 u + 4 mq + e)

@@ -868,8 +868,8 @@ def row_tiles_faster(rows: "tuple[int, ...] | list[int]", lengths: "tuple[int, .
     key/value heads, GQA 1 to 8, every head width) and checked on 950 others, each measured both
     ways: 500 prompts, chunks, windows and mixed steps of the usual head shapes, on which the choice
     takes 0.9% more than the faster side on average, and 450 of many short requests, 2.7%. It takes
-    tiles where row by row is more than 5% faster on 21 of them (the worst: 251 requests of 3 rows,
-    64/32 heads of 64, 177 and 121 us), and rows where tiles are on 44 (the worst: one key/value
+    tiles where row by row is more than 5% faster on 21 of them (the worst: a chunk of 457 rows beside
+    250 requests of 1 or 2, 64/32 heads of 64, 177 and 121 us), and rows where tiles are on 44 (the worst: one key/value
     head, whose rows it under-prices: 226 rows, 8 heads of 128, 160 and 70 us).
     """
     counts = np.array(rows, dtype=np.int64)

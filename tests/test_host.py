@@ -376,6 +376,7 @@ def test_fp32_row_tiles_choice() -> None:
         (([4] * 64, [1000] * 64), (9, 3, 64), (75.7, 35.8)),  # windows
         (([8] * 60, [600] * 60), (16, 8, 256), (721, 112)),
         (([256] + [1] * 30, [1000] + [500] * 30), (64, 8, 128), (335, 156)),  # a chunk beside decode rows
+        (([22, 1], [94, 100]), (32, 8, 64), (14.8, 10.1)),  # near the line
         (([1] * 512, [128] * 512), (9, 3, 64), (18.1, 54.5)),  # one-row requests: a tile walks up to 11 of them
         (([1] * 512, [1024] * 512), (32, 4, 64), (185, 229)),
         (([1] * 256, [128] * 256), (32, 8, 64), (23.2, 39.0)),
