@@ -819,6 +819,9 @@ ROWS_WIDE_FIXED, ROWS_WIDE_RATE = 1.5, 0.775
 #: The tiles are taken up to this ratio of the modelled times: the median of tiles modelled over tiles
 #: measured is 1.11 (950 steps; a ratio of 1 costs 2.4% over the faster side on them, 1.1 1.8%).
 ROW_TILES_MARGIN = 1.1
+#: Steps of up to this many requests are first decided by bounds in a loop over the requests (about 1.5 us
+#: each, most steps), the others and the rest by listing the tiles in numpy (40 us and more).
+ROW_TILES_BOUND_REQUESTS = 24
 
 
 def row_tile_shape(n_rows: int, num_kv_heads: int, group: int, head_dim: int) -> tuple[int, int]:
@@ -856,6 +859,47 @@ def row_tile_walks(rows: np.ndarray, lengths: np.ndarray, group: int, pairs: int
     return np.bincount(tile), np.bincount(tile, weights=steps)
 
 
+def row_tiles_busy_bounds(rows: "tuple[int, ...] | list[int]", lengths: "tuple[int, ...] | list[int]", group: int,
+                          pairs: int, waves: int, slots: int, per_request: float, per_step: float
+                          ) -> tuple[float, float]:
+    """Bounds of the finish time of a step's tiles (:func:`row_tile_walks`, ``per_request`` and
+    ``per_step`` us each) over ``slots`` compute units, without listing them: the longest tile, exactly,
+    and the sum of all, from the mean position at which a request's inner tiles end."""
+    step = 16 * waves
+    total = spare = longest = shared = 0.0  # shared: the last tile's time so far
+    start, open_tile = 0, -1
+    for count, length in zip(rows, lengths):
+        if not count:
+            continue
+        unit = per_step if length else 0.0
+        end = start + count * group
+        first, last = start // pairs, (end - 1) // pairs
+        before = length - count
+        time = per_request + unit * ((length - 1) // step + 1)  # of the request's last tile
+        total += time
+        carried = shared if first == open_tile else 0.0
+        if first == last:
+            shared = carried + time
+        else:
+            shared = time
+            time = per_request + unit * ((before + (first * pairs + pairs - 1 - start) // group) // step + 1)
+            total += time
+            longest = max(longest, carried + time)
+            inner = last - first - 1
+            if inner:
+                time = per_request + unit * ((before + (last * pairs - 1 - start) // group) // step + 1)
+                longest = max(longest, time)
+                # steps(t) = floor(x(t) / step) + 1, x(t) even over the inner tiles
+                mean = before + (((first + last) / 2 + 1) * pairs - 1 - start) / group
+                total += inner * (per_request + unit * mean / step)
+                spare += inner * unit
+        longest = max(longest, shared)
+        start, open_tile = end, last
+    if open_tile < slots:
+        return longest, longest
+    return max(longest, total / slots), longest + (total + spare) / slots
+
+
 def row_tiles_faster(rows: "tuple[int, ...] | list[int]", lengths: "tuple[int, ...] | list[int]", num_kv_heads: int,
                      group: int, head_dim: int) -> bool:
     """Whether an fp32 multi-row step of ``rows`` query rows over contexts of ``lengths`` per request
@@ -872,6 +916,29 @@ def row_tiles_faster(rows: "tuple[int, ...] | list[int]", lengths: "tuple[int, .
     250 requests of 1 or 2, 64/32 heads of 64, 177 and 121 us), and rows where tiles are on 44 (the worst: one key/value
     head, whose rows it under-prices: 226 rows, 8 heads of 128, 160 and 70 us).
     """
+    wide = group // head_chunks(group) == 8
+    row_bytes = num_kv_heads * 2 * head_dim * 4
+    slots = max(1, COMPUTE_UNITS // num_kv_heads)  # a tile runs once per key/value head, side by side
+    pairs, waves = row_tile_shape(sum(rows), num_kv_heads, group, head_dim)
+    fixed, per_request, per_step = ROW_TILES_US[(head_dim, pairs // 16)]
+
+    def most(positions: int) -> float:  # the tiles' time up to which they are taken
+        by_row = (ROWS_FIXED_US[head_dim] * (ROWS_WIDE_FIXED if wide else 1.0)
+                  + positions * row_bytes / (ROWS_BYTES_PER_US * (ROWS_WIDE_RATE if wide else 1.0)))
+        return by_row * ROW_TILES_MARGIN - fixed
+
+    if len(rows) <= ROW_TILES_BOUND_REQUESTS:
+        positions = contexts = 0
+        for count, length in zip(rows, lengths):
+            if count and length:
+                positions += count * (2 * length - count + 1) // 2
+                contexts += length
+        if not positions:
+            return False
+        limit, stream = most(positions), contexts * row_bytes / ROW_TILES_BYTES_PER_US
+        low, high = row_tiles_busy_bounds(rows, lengths, group, pairs, waves, slots, per_request, per_step)
+        if max(high, stream) < limit or max(low, stream) >= limit:
+            return max(high, stream) < limit
     counts = np.array(rows, dtype=np.int64)
     contexts = np.array(lengths, dtype=np.int64)
     if not counts.all():  # requests without rows hold no pairs
@@ -880,18 +947,9 @@ def row_tiles_faster(rows: "tuple[int, ...] | list[int]", lengths: "tuple[int, .
     positions = int(seen.dot(2 * contexts - seen + 1)) // 2  # of all rows' contexts
     if not positions:
         return False
-    row_bytes = num_kv_heads * 2 * head_dim * 4
-    wide = group // head_chunks(group) == 8
-    by_row = (ROWS_FIXED_US[head_dim] * (ROWS_WIDE_FIXED if wide else 1.0)
-              + positions * row_bytes / (ROWS_BYTES_PER_US * (ROWS_WIDE_RATE if wide else 1.0)))
-    pairs, waves = row_tile_shape(int(counts.sum()), num_kv_heads, group, head_dim)
-    fixed, per_request, per_step = ROW_TILES_US[(head_dim, pairs // 16)]
     tile, steps = _row_tile_steps(counts, contexts, group, pairs, waves)
-    # a tile runs once per key/value head: that many workgroups of its length side by side
-    busy = _dispatch_makespan(np.bincount(tile, weights=per_step * steps + per_request),
-                              max(1, COMPUTE_UNITS // num_kv_heads))
-    tiles = fixed + max(busy, int(contexts.sum()) * row_bytes / ROW_TILES_BYTES_PER_US)
-    return tiles < by_row * ROW_TILES_MARGIN
+    busy = _dispatch_makespan(np.bincount(tile, weights=per_step * steps + per_request), slots)
+    return max(busy, int(contexts.sum()) * row_bytes / ROW_TILES_BYTES_PER_US) < most(positions)
 
 
 def choose_prefill_partition(group_lengths: list[int], row_lengths: tuple[int, ...] | list[int],

@@ -415,6 +415,26 @@ def test_fp32_row_tiles_walk_their_requests_one_by_one() -> None:
             steps.append(sum(-(-n // (16 * waves)) for n in longest.values()))
         got = hip_attention.row_tile_walks(rows, lengths, group, pairs, waves)
         assert got[0].tolist() == requests and got[1].tolist() == steps, case
+        # the bounds that decide most steps hold the scheduled time (requests without rows among them)
+        some = [(0, 7), *zip(rows.tolist(), lengths.tolist()), (0, 0)]
+        for slots in (1, 8, 256):
+            low, high = hip_attention.row_tiles_busy_bounds(*zip(*some), group, pairs, waves, slots, 2.7, 1.7)
+            busy = hip_attention._dispatch_makespan(2.7 * got[0] + 1.7 * got[1], slots)
+            assert low <= busy * (1 + 1e-12) and busy <= high * (1 + 1e-12), (case, slots)
+
+
+def test_fp32_row_tiles_choice_by_bounds_is_the_scheduled_one(monkeypatch: pytest.MonkeyPatch) -> None:
+    rng = np.random.default_rng(92)
+    steps = []
+    for _ in range(150):
+        rows = rng.integers(0, rng.choice([2, 9, 300]), size=int(rng.integers(1, 25)))
+        lengths = np.where(rng.random(rows.size) < 0.1, 0, rows + rng.integers(0, rng.choice([50, 3000]), size=rows.size))
+        steps.append((rows.tolist(), lengths.tolist(), int(rng.choice([1, 3, 8, 32])), int(rng.integers(1, 17)),
+                      int(rng.choice([64, 128, 256]))))
+    chosen = [hip_attention.row_tiles_faster(*step) for step in steps]
+    monkeypatch.setattr(hip_attention, "ROW_TILES_BOUND_REQUESTS", 0)
+    assert [hip_attention.row_tiles_faster(*step) for step in steps] == chosen
+    assert any(chosen) and not all(chosen)
 
 
 def test_multi_row_launch_choice_by_head_width() -> None:
